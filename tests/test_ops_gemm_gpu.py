@@ -101,6 +101,27 @@ def test_non_finite_operands(dev, M, K, N):
         assert rel(a[ok], e[ok]) < tol(K)
 
 
+@pytest.mark.parametrize("row,col", [(None, 0), (None, 31), (None, 45), (0, None), (17, None), (63, None)])
+def test_second_pass_where_few_lanes_overflow(dev, row, col):
+    """A value beyond bf16's largest in one row or one column only, so that most
+    lanes of a wave (the first among them, or not) have finite sums."""
+    import torch
+
+    M, K, N = 64, 768, 768
+    g = torch.Generator(device=dev).manual_seed(11)
+    x, w = (torch.empty(s, device=dev).normal_(0.0, 1.0, generator=g) for s in ((M, K), (K, N)))
+    b, y = torch.zeros(N, device=dev), torch.empty((M, N), device=dev)
+    if col is None:
+        x[row, 300], w[300] = 3.4e38, w[300] * 1e-37
+    else:
+        w[300, col], x[:, 300] = -3.4e38, x[:, 300] * 1e-37
+    ops.device_linear_activation_fused_forward(y, None, x, w, b, False, 1, M, K, N)
+    r = x.double() @ w.double()
+    assert torch.isfinite(y).all()
+    part = (slice(None), col) if row is None else row
+    assert rel(y, r) < tol(K) and rel(y[part], r[part]) < tol(K)
+
+
 def test_captured_products_replay(dev):
     """A captured linear layer (which takes no split-k workspace) replayed
     between eager calls gives the eager results' values, and the same bits on
