@@ -25,7 +25,8 @@
  *   - Matrix products take fp32 operands whole: the library's own kernel
  *     holds each as three bf16 terms (24 significand bits), multiplies those on
  *     the bf16 matrix cores and accumulates in fp32 (the reference's CUDA
- *     backend uses TF32 tensor cores); rows that are not 16-byte aligned
+ *     backend uses TF32 tensor cores), or, where an operand is not finite or a
+ *     row below 2^-95, on the fp32 matrix cores; rows that are not 16-byte aligned
  *     multiples of 4 floats, and sizes where they are faster, go to
  *     hipBLASLt / rocBLAS fp32 GEMMs. The
  *     element-wise, normalisation and reduction work runs on this library's

@@ -149,3 +149,35 @@ def test_captured_products_replay(dev):
     ops.release_workspaces()
     ops.device_linear_activation_fused_forward(e, None, x, w, b, False, 1, M, K, N)
     assert rel(e, x.double() @ w.double()) < tol(K)
+
+
+@pytest.mark.parametrize("M,K,N", [(77, 768, 768), (2050, 768, 2304)])
+@pytest.mark.parametrize("e", [94, 112, 118, 124])
+def test_tiny_operands(dev, M, K, N, e):
+    """Operands of 2^-e, where bf16 terms are subnormal: all of them, and one
+    row or column among ordinary ones, keep the precision of an fp32 product."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(e)
+
+    def rnd(*s, std=1.0):
+        return torch.empty(s, device=dev).normal_(0.0, std, generator=g)
+
+    x, w, gy, b, y = rnd(M, K), rnd(K, N), rnd(M, N), torch.zeros(N, device=dev), torch.empty((M, N), device=dev)
+    small = 2.0 ** -e
+    xt, wt, gt = x.clone(), w.clone(), gy * small
+    xt[M // 2] *= small
+    wt[:, N // 3] *= small
+    xz, wz = xt.clone(), wt.clone()  # the first k zeros
+    xz[:, :40] = 0
+    wz[:40] = 0
+    for a, c in ((x * small, w), (x, w * small), (xt, w), (x, wt), (xz, w), (x, wz)):
+        ops.device_linear_activation_fused_forward(y, None, a, c, b, False, 1, M, K, N)
+        r = a.double() @ c.double()
+        assert rel(y, r) < tol(K)
+        assert rel(y[M // 2], r[M // 2]) < tol(K)
+        assert rel(y[:, N // 3], r[:, N // 3]) < tol(K)
+    gx, gw, gb = torch.empty((M, K), device=dev), torch.zeros((K, N), device=dev), torch.zeros(N, device=dev)
+    ops.device_linear_backward(gx, gw, gb, gt, x, w, 1, M, K, N)
+    assert rel(gx, gt.double() @ w.double().t()) < tol(N)
+    assert rel(gw, x.double().t() @ gt.double()) < tol(M)
