@@ -21,6 +21,7 @@
 #include "attn_common.h"
 #include "attn_kernels.h"
 
+#include <float.h>
 #include <type_traits>
 
 namespace gpt_attn {
@@ -149,14 +150,16 @@ template <int ND> __device__ __forceinline__ void add_cols(v4f (&acc)[ND], const
 
 // Merges the waves' accumulators (each times `mine`, its factor for the lane's
 // row l16) through `red` (kMerge floats), wave w writing register w of every
-// accumulator to out[row l16][dimension].
+// accumulator to out[row l16][dimension]. Returns whether a value that this
+// lane stored is not finite.
 constexpr int kMergeN = 8, kMerge = kWaves * kMergeN * 4 * 64;
 template <int ND, bool VEC>
-__device__ __forceinline__ void merge_store(const v4f (&acc)[ND], float mine, float *red, float *out, long W, int d,
+__device__ __forceinline__ bool merge_store(const v4f (&acc)[ND], float mine, float *red, float *out, long W, int d,
                                             bool row_ok, int w, int lane)
 {
     constexpr int NU = Head<ND>::NU;
     const int l16 = lane & 15, kc = lane >> 4;
+    bool bad = false;
 #pragma unroll
     for (int n0 = 0; n0 < ND; n0 += kMergeN)
     {
@@ -186,6 +189,9 @@ __device__ __forceinline__ void merge_store(const v4f (&acc)[ND], float mine, fl
                 float *const dst = out + l16 * W + e;
                 if (row_ok)
                 {
+#pragma unroll
+                    for (int u = 0; u < NU; ++u)
+                        bad |= !__builtin_isfinite(o[u]);
                     if (VEC && NU == 4)
                     {
                         if (e < d)
@@ -201,6 +207,154 @@ __device__ __forceinline__ void merge_store(const v4f (&acc)[ND], float mine, fl
                 }
             }
     }
+    return bad;
+}
+
+// Whether x holds in any lane of the workgroup (through red: __syncthreads_or has
+// LDS of its own, with which five backward workgroups no longer fit a CU).
+__device__ __forceinline__ bool any_lane(bool x, float *red, int w, int lane)
+{
+    x = __any(x);
+    __syncthreads();
+    if (lane == 0)
+        red[w] = x ? 1.f : 0.f;
+    __syncthreads();
+    return red[0] + red[1] + red[2] + red[3] != 0.f;
+}
+
+// The matrix products above multiply a masked pair's weight of 0 with what
+// stands in its rows: an infinity or NaN in V or K of a key after the query, or in
+// Q or dO of a query before the key, would reach results of the same diagonal
+// block, and a wave whose blocks hold no score but -inf has no maximum to take them
+// against. A workgroup with an output that is not finite therefore works its rows
+// out again, pair by pair: 16 lanes a row, lane p dimensions p + 16 u, over the
+// row's own keys (or queries) alone.
+template <int ND> struct Pairs
+{
+    int g, p;  // row of the block, lane of the row
+    int d;
+    __device__ __forceinline__ explicit Pairs(int dims) : d(dims)
+    {
+        int t = (int)threadIdx.x;
+        asm volatile("" : "+v"(t));  // shares nothing with the first pass, whose registers it would hold
+        g = t >> 4;
+        p = t & 15;
+    }
+    __device__ __forceinline__ void load(float (&f)[ND], const float *row) const
+    {
+#pragma unroll
+        for (int u = 0; u < ND; ++u)
+            f[u] = p + 16 * u < d ? row[p + 16 * u] : 0.f;
+    }
+    __device__ __forceinline__ void store(float *row, const float (&f)[ND], float scale) const
+    {
+#pragma unroll
+        for (int u = 0; u < ND; ++u)
+            if (p + 16 * u < d)
+                row[p + 16 * u] = f[u] * scale;
+    }
+    static __device__ __forceinline__ float dot(const float (&a)[ND], const float (&b)[ND])
+    {
+        float x = 0.f;
+#pragma unroll
+        for (int u = 0; u < ND; ++u)
+            x += a[u] * b[u];
+        return row16_sum(x);
+    }
+    static __device__ __forceinline__ void add(float (&acc)[ND], float w, const float (&b)[ND])
+    {
+#pragma unroll
+        for (int u = 0; u < ND; ++u)
+            acc[u] += w * b[u];
+    }
+};
+
+template <int ND>
+__device__ __forceinline__ void fwd_pairs(float *y, float *lse, const float *x, int T, long C, int H, int b, int h, int q0, int d,
+                                          float qscale)
+{
+    const Pairs<ND> pr(d);
+    const int i = q0 + pr.g;
+    if (i >= T)
+        return;
+    const float *const base = x + (long)b * T * 3 * C + (long)h * d;
+    float q[ND], o[ND] = {}, m = -FLT_MAX, l = 0.f;
+    pr.load(q, base + (long)i * 3 * C);
+#pragma unroll 1
+    for (int j = 0; j <= i; ++j)
+    {
+        float k[ND], v[ND];
+        pr.load(k, base + (long)j * 3 * C + C);
+        pr.load(v, base + (long)j * 3 * C + 2 * C);
+        const float s = Pairs<ND>::dot(q, k) * qscale, mn = fmaxf(m, s), corr = fast_exp2(m - mn), e = fast_exp2(s - mn);
+        m = mn;
+        l = l * corr + e;
+#pragma unroll
+        for (int u = 0; u < ND; ++u)
+            o[u] = o[u] * corr + e * v[u];
+    }
+    pr.store(y + ((long)b * T + i) * C + (long)h * d, o, 1.f / l);
+    if (pr.p == 0)
+        lse[((long)b * T + i) * H + h] = (m + fast_log2(l)) * kLn2;
+}
+
+template <int ND>
+__device__ __forceinline__ void dq_pairs(float *gx, const float *lse, const float *dy, const float *y, const float *x, int T,
+                                         long C, int H, int b, int h, int q0, int d, float scale, float qscale)
+{
+    const Pairs<ND> pr(d);
+    const int i = q0 + pr.g;
+    if (i >= T)
+        return;
+    const float *const base = x + (long)b * T * 3 * C + (long)h * d;
+    const long at = ((long)b * T + i) * C + (long)h * d;
+    float q[ND], g[ND], acc[ND] = {}, D;
+    pr.load(q, base + (long)i * 3 * C);
+    pr.load(g, dy + at);
+    {
+        float o[ND];
+        pr.load(o, y + at);
+        D = Pairs<ND>::dot(g, o);
+    }
+    const float L = lse[((long)b * T + i) * H + h] * kLog2e;
+#pragma unroll 1
+    for (int j = 0; j <= i; ++j)
+    {
+        float k[ND], v[ND];
+        pr.load(k, base + (long)j * 3 * C + C);
+        pr.load(v, base + (long)j * 3 * C + 2 * C);
+        const float e = fast_exp2(Pairs<ND>::dot(q, k) * qscale - L);
+        Pairs<ND>::add(acc, e * (Pairs<ND>::dot(g, v) - D), k);
+    }
+    pr.store(gx + ((long)b * T + i) * 3 * C + (long)h * d, acc, scale);
+}
+
+template <int ND>
+__device__ __forceinline__ void dkdv_pairs(float *gx, const float *lse, const float *D, const float *dy, const float *x, int T,
+                                           long C, int H, int b, int h, int k0, int d, float scale, float qscale)
+{
+    const Pairs<ND> pr(d);
+    const int j = k0 + pr.g;
+    if (j >= T)
+        return;
+    const float *const base = x + (long)b * T * 3 * C + (long)h * d;
+    float k[ND], v[ND], dk[ND] = {}, dv[ND] = {};
+    pr.load(k, base + (long)j * 3 * C + C);
+    pr.load(v, base + (long)j * 3 * C + 2 * C);
+#pragma unroll 1
+    for (int i = j; i < T; ++i)
+    {
+        float q[ND], g[ND];
+        pr.load(q, base + (long)i * 3 * C);
+        pr.load(g, dy + ((long)b * T + i) * C + (long)h * d);
+        const long at = ((long)b * T + i) * H + h;
+        const float e = fast_exp2(Pairs<ND>::dot(q, k) * qscale - lse[at] * kLog2e);
+        Pairs<ND>::add(dk, e * (Pairs<ND>::dot(g, v) - D[at]), q);
+        Pairs<ND>::add(dv, e, g);
+    }
+    float *const out = gx + ((long)b * T + j) * 3 * C + (long)h * d;
+    pr.store(out + C, dk, scale);
+    pr.store(out + 2 * C, dv, 1.f);
 }
 
 // Workgroup -> (b, h) and row block: (b, h) fastest, so that with B H a
@@ -234,6 +388,18 @@ __global__ __launch_bounds__(64 * kWaves, ND <= 8 ? 2 : 1) void fwd_general_kern
     const long W = 3L * C;
     const float *const base = qkv + (long)it.b * T * W + (long)it.h * d;
     const int q0 = kRows * it.blk;
+    // What a second pass would need, for the 4-byte form, whose loops spill scalar
+    // registers as it is (B = 2, T = 200, H = 4, d = 129: 50.9 us, 55.1 with them held).
+    struct Held
+    {
+        float *y, *lse;
+        const float *qkv;
+        int T, C, H, b, h, q0, d;
+        float qscale;
+    };
+    __shared__ Held held;
+    if (!VEC && threadIdx.x == 0)
+        held = Held{y, lse, qkv, T, C, H, it.b, it.h, q0, d, qscale};
 
     float q[ND][4];
     load_rows<ND, VEC>(q, rows_of(base, q0, T, W, d), d, l16, kc);
@@ -293,10 +459,17 @@ __global__ __launch_bounds__(64 * kWaves, ND <= 8 ? 2 : 1) void fwd_general_kern
     for (int k = 0; k < kWaves; ++k)
         L += sl[k][l16] * fast_exp2(sm[k][l16] - M);
     const int row = q0 + l16;
-    merge_store<ND, VEC>(acc, fast_exp2(m - M) / L, red, y + ((long)it.b * T + q0) * C + (long)it.h * d, C, d, row < T, w,
-                         lane);
+    const bool bad = merge_store<ND, VEC>(acc, fast_exp2(m - M) / L, red, y + ((long)it.b * T + q0) * C + (long)it.h * d, C, d,
+                                         row < T, w, lane);
     if (w == 0 && kc == 0 && row < T)
         lse[((long)it.b * T + row) * H + it.h] = (M + fast_log2(L)) * kLn2;
+    if (any_lane(bad, red, w, lane))
+    {
+        if (VEC)
+            fwd_pairs<ND>(y, lse, qkv, T, C, H, it.b, it.h, q0, d, qscale);
+        else
+            fwd_pairs<ND>(held.y, held.lse, held.qkv, held.T, held.C, held.H, held.b, held.h, held.q0, held.d, held.qscale);
+    }
 }
 
 // D and dQ of 16 queries (lane: query l16, keys 4 kc + r).
@@ -360,7 +533,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void bwd_dq_general_kernel(float *_
         }
         add_cols<ND>(acc, kt, ds);
     }
-    merge_store<ND, VEC>(acc, scale, red, grad_x + ((long)it.b * T + q0) * W + (long)it.h * d, W, d, row < T, w, lane);
+    const bool bad =
+        merge_store<ND, VEC>(acc, scale, red, grad_x + ((long)it.b * T + q0) * W + (long)it.h * d, W, d, row < T, w, lane);
+    if (any_lane(bad, red, w, lane))
+        dq_pairs<ND>(grad_x, lse, dy, y, qkv, T, C, H, it.b, it.h, q0, d, scale, qscale);
 }
 
 // dK and dV of 16 keys (lane: key l16, queries 4 kc + r). The keys' own rows
@@ -435,8 +611,10 @@ __global__ __launch_bounds__(64 * kWaves, 1) void bwd_dkdv_general_kernel(float 
         }
     }
     float *const out = grad_x + ((long)it.b * T + k0) * W + (long)it.h * d;
-    merge_store<ND, VEC>(dk, scale, red, out + C, W, d, k0 + l16 < T, w, lane);
-    merge_store<ND, VEC>(dv, 1.f, red, out + 2L * C, W, d, k0 + l16 < T, w, lane);
+    bool bad = merge_store<ND, VEC>(dk, scale, red, out + C, W, d, k0 + l16 < T, w, lane);
+    bad |= merge_store<ND, VEC>(dv, 1.f, red, out + 2L * C, W, d, k0 + l16 < T, w, lane);
+    if (any_lane(bad, red, w, lane))
+        dkdv_pairs<ND>(grad_x, lse, D, dy, qkv, T, C, H, it.b, it.h, k0, d, scale, qscale);
 }
 
 bool vec_ok(const Shape &s, const void *a, const void *b, const void *c, const void *e = nullptr)

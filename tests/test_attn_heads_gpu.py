@@ -77,6 +77,64 @@ def test_misaligned_pointers(dev, d):
     run(dev, 2, 70, 2, d, off=1)
 
 
+def pairs64(x, gy, T, d):
+    """y, dq, dk, dv and lse of one head in float64, every query over its own keys
+    alone, so that no value meets a masked one."""
+    q, k, v = x.double().unbind(1)
+    g, sc = gy.double(), d ** -0.5
+    y, dq, dk, dv = (np.zeros((T, d)) for _ in range(4))
+    lse = np.zeros(T)
+    q, k, v, g = (t.cpu().numpy() for t in (q, k, v, g))
+    with np.errstate(all="ignore"):
+        for i in range(T):
+            s = (k[:i + 1] * q[i]).sum(1) * sc
+            m = np.nanmax(s) if np.isfinite(s).any() else 0.0
+            e = np.exp(s - m)
+            p = e / e.sum()
+            lse[i] = m + np.log(e.sum())
+            y[i] = (p[:, None] * v[:i + 1]).sum(0)
+            ds = p * ((v[:i + 1] * g[i]).sum(1) - (y[i] * g[i]).sum()) * sc
+            dq[i] = (ds[:, None] * k[:i + 1]).sum(0)
+            dk[:i + 1] += ds[:, None] * q[i]
+            dv[:i + 1] += p[:, None] * g[i]
+    return {"y": y, "lse": lse, "dq": dq, "dk": dk, "dv": dv}
+
+
+@pytest.mark.parametrize("d", [16, 20, 33, 128, 250])
+@pytest.mark.parametrize("what", ["k", "v", "q", "g", "low"])
+@pytest.mark.parametrize("row", [5, 20, 37])
+def test_non_finite_values_stay_with_their_pairs(dev, d, what, row):
+    """An infinity or NaN reaches the rows that causality gives it and no others of
+    their 16-row blocks; scores of -infinity (low) weigh nothing."""
+    import torch
+
+    T, H = 40, 2
+    C = H * d
+    g = torch.Generator(device=dev).manual_seed(d + row)
+    x = torch.empty((1, T, 3, H, d), device=dev).normal_(generator=g)
+    gy = torch.empty((1, T, H, d), device=dev).normal_(generator=g)
+    if what == "g":
+        gy[0, row, 1, 1] = np.nan
+    elif what == "low":
+        x[0, :, 0, 1, 0], x[0, :, 1, 1, 0] = 1e25, 0.0
+        x[0, 16:32, 1, 1, 0] = x[0, row + 1, 1, 1, 0] = -1e25
+    else:
+        x[0, row, "qkv".index(what), 1, 1] = np.inf if what == "v" else np.nan
+    y, lse, gx, D = (torch.empty(s, device=dev) for s in ((1, T, C), (1, T, H), (1, T, 3 * C), (1, T, H)))
+    gpt_amd.device_flash_attention_forward(y, lse, x, 1, T, C, H)
+    gpt_amd.device_flash_attention_backward(gx, D, lse, gy, y, x, 1, T, C, H)
+    for h in range(H):
+        r = pairs64(x[0, :, :, h], gy[0, :, h], T, d)
+        o = gx.view(T, 3, H, d)[:, :, h]
+        a = {"y": y.view(T, H, d)[:, h], "lse": lse.view(T, H)[:, h], "dq": o[:, 0], "dk": o[:, 1], "dv": o[:, 2]}
+        for name, t in a.items():
+            t, e = t.double().cpu().numpy(), r[name]
+            ok = np.isfinite(e)
+            assert np.array_equal(np.isfinite(t), ok), (name, h)
+            if ok.any():
+                assert np.abs(t[ok] - e[ok]).max() <= TOL * max(np.abs(e[ok]).max(), 1e-3), (name, h)
+
+
 def test_rows_beyond_buffer_offsets_and_one_grid_dimension(dev):
     """16 rows of 400 MB each are past a buffer range's 31-bit offsets, and one
     workgroup per head is more than a launch dimension takes."""

@@ -213,3 +213,108 @@ def test_forward_output_rows_are_written_through():
                 assert not plain, (name, plain[:4])
                 found += 1
     assert found == 1
+
+
+# Wait states that an MFMA's result takes until another instruction may read it
+# (passes + 2 for fp32, + 4 for the bf16 one).
+MFMA_READ_WAIT = {"v_mfma_f32_16x16x4_f32": 10, "v_mfma_f32_32x32x2_f32": 18, "v_mfma_f32_16x16x32_bf16": 8}
+
+
+def av_regs(tok):
+    tok = tok.strip().split()[0].strip("-|")
+    m = re.fullmatch(r"([av])\[(\d+):(\d+)\]", tok)
+    if m:
+        return {(m.group(1), k) for k in range(int(m.group(2)), int(m.group(3)) + 1)}
+    m = re.fullmatch(r"([av])(\d+)", tok)
+    return {(m.group(1), int(m.group(2)))} if m else set()
+
+
+def early_mfma_reads(asm):
+    """Reads of an MFMA's result by other instructions, along every branch, before
+    it is there. The compiler keeps the distance within a block, but was seen to
+    leave the wait out where a branch stands between the two (an experimental
+    kernel, never shipped: the read came after 2 to 6 wait states of 10 and returned
+    the register's old value)."""
+    found, n = [], 0
+    funcs, cur = [], None
+    for line in asm.splitlines():
+        m = re.match(r"^[0-9a-f]+ <(\S+)>:", line)
+        if m:
+            cur = []
+            funcs.append((m.group(1), cur))
+            continue
+        m = re.match(r"^\s+(\S.*?)\s*//\s*([0-9A-F]+):(.*)", line)
+        if cur is not None and m:
+            t = re.search(r"<\S+\+0x([0-9a-f]+)>", m.group(3))
+            cur.append((int(m.group(2), 16), m.group(1), int(t.group(1), 16) if t else None))
+    for name, ins in funcs:
+        where = {a: i for i, (a, _, _) in enumerate(ins)}
+        for i, (_, s, _) in enumerate(ins):
+            if not s.startswith("v_mfma"):
+                continue
+            n += 1
+            op, rest = s.split(None, 1)
+            need = MFMA_READ_WAIT[op]
+            paths, seen = [(i + 1, 0, frozenset(av_regs(rest.split(",")[0])))], set()
+            while paths:
+                j, w, live = paths.pop()
+                while w < need and j < len(ins) and live and (j, w, live) not in seen:
+                    seen.add((j, w, live))
+                    _, t, target = ins[j]
+                    op2, _, args = t.partition(" ")
+                    ops = [av_regs(o) for o in args.split(",")] if args.strip() else []
+                    if op2.startswith("v_mfma"):
+                        live -= ops[0]
+                    elif op2.startswith("v_"):
+                        if live & set().union(*ops[1:]):
+                            found.append(f"{name}: {s}  ->  {t} after {w} of {need}")
+                            break
+                        live -= ops[0]
+                    elif re.match(r"(ds|buffer|global|flat|scratch)_", op2) and ops and live & set().union(*ops):
+                        if "store" in op2 or "write" in op2 or "permute" in op2 or live & set().union(*ops[1:]):
+                            found.append(f"{name}: {s}  ->  {t} after {w} of {need}")
+                            break
+                    w += int(args, 0) + 1 if op2 == "s_nop" else 1
+                    if "branch" in op2 and target is not None:
+                        k = where.get(ins[0][0] + target)
+                        if k is not None:
+                            paths.append((k, w, live))
+                    if op2 in ("s_branch", "s_endpgm"):
+                        break
+                    j += 1
+    return n, found
+
+
+@pytest.mark.parametrize("lib", LIBS, ids=os.path.basename)
+def test_no_mfma_result_read_early(lib, tmp_path):
+    if not os.path.exists(lib):
+        pytest.skip("library not built")
+    n_mfma, bad = 0, []
+    for k, obj in enumerate(gfx950_code_objects(lib)):
+        f = tmp_path / f"co{k}.o"
+        f.write_bytes(obj)
+        asm = subprocess.run([OBJDUMP, "-d", "--mcpu=gfx950", str(f)], capture_output=True, text=True,
+                             check=True).stdout
+        n, found = early_mfma_reads(asm)
+        n_mfma += n
+        bad += found
+    assert n_mfma > 0
+    assert not bad, "\n".join(bad[:20])
+
+
+def test_mfma_read_scanner():
+    """A read behind a branch, one after enough wait states, one of another register."""
+    head = "0000000000001000 <k>:\n"
+    lines = ["v_mfma_f32_16x16x4_f32 a[8:11], v35, v9, a[16:19]", "v_add_f32_e32 v1, v2, v3", "s_cbranch_vccnz 2",
+             "s_nop 9", "s_nop 0", "v_accvgpr_read_b32 v33, a11", "s_endpgm"]
+
+    def text(ls, target):
+        out = head
+        for k, l in enumerate(ls):
+            out += f"\t{l} // {0x1000 + 8 * k:012X}: 00000000" + (f" <k+0x{8 * target:x}>" if "branch" in l else "") + "\n"
+        return out
+
+    assert len(early_mfma_reads(text(lines, 5))[1]) == 1   # the branch skips the wait
+    assert early_mfma_reads(text(lines, 3))[1] == []
+    assert early_mfma_reads(text([l.replace("a11", "a12") for l in lines], 5))[1] == []
+    assert len(early_mfma_reads(text(["v_mfma_f32_16x16x4_f32 v[0:3], v35, v9, v[0:3]", "ds_write_b32 v9, v2"], 0))[1]) == 1
