@@ -14,6 +14,7 @@
 #include <hipblaslt/hipblaslt.h>
 #include <rocblas/rocblas.h>
 
+#include <atomic>
 #include <math.h>
 #include <mutex>
 #include <stdarg.h>
@@ -379,27 +380,44 @@ int lt_gemm(const char *op, hipStream_t st, bool ta, bool tb, int M, int N, int 
 
 bool use_lt(bool ta, int N) { return ta || N <= 1024; }
 
-// Shapes that the library's own kernel has been considered for, with their launch choices.
+// Shapes that the library's own kernel has been considered for, with their launch
+// choices, and whether one has been launched. Entries stay where they are; past
+// kOwnFull shapes choices are made anew for each call, and not counted.
 struct OwnPlan
 {
     int M, N, K;
     bool ta, tb;
+    std::atomic<bool> ran;
     gpt_ops::gemm::Choice c;
 };
+constexpr int kOwnPlans = 1024, kOwnFull = 768;
 std::mutex g_own_mu;
-OwnPlan g_own[kMaxPlans];
+OwnPlan g_own[kOwnPlans];  // K = 0: free; a shape's entry is at its hash or after
 int g_nown = 0;
+std::atomic<int> g_own_ran{0};
 
-gpt_ops::gemm::Choice own_choice(int M, int N, int K, bool ta, bool tb)
+// The plan of a shape; `spare` where the table is full.
+OwnPlan *own_plan(int M, int N, int K, bool ta, bool tb, OwnPlan *spare)
 {
     std::lock_guard<std::mutex> lock(g_own_mu);
-    for (int i = 0; i < g_nown; ++i)
-        if (g_own[i].M == M && g_own[i].N == N && g_own[i].K == K && g_own[i].ta == ta && g_own[i].tb == tb)
-            return g_own[i].c;
-    const gpt_ops::gemm::Choice c = gpt_ops::gemm::choose(M, N, K, ta, tb, true);
-    if (g_nown < kMaxPlans)
-        g_own[g_nown++] = OwnPlan{M, N, K, ta, tb, c};
-    return c;
+    unsigned h = ((unsigned)M * 0x9E3779B1u) ^ ((unsigned)N * 0x85EBCA77u) ^ ((unsigned)K * 0xC2B2AE3Du) ^ (ta ? 1u : 0u) ^ (tb ? 2u : 0u);
+    h = (h ^ h >> 15) % kOwnPlans;
+    for (; g_own[h].K; h = (h + 1) % kOwnPlans)
+    {
+        OwnPlan &p = g_own[h];
+        if (p.M == M && p.N == N && p.K == K && p.ta == ta && p.tb == tb)
+            return &p;
+    }
+    OwnPlan *p = spare;
+    if (g_nown < kOwnFull)
+    {
+        p = &g_own[h];
+        ++g_nown;
+    }
+    p->M = M, p->N = N, p->K = K, p->ta = ta, p->tb = tb;
+    p->ran = p == spare;
+    p->c = gpt_ops::gemm::choose(M, N, K, ta, tb, true);
+    return p;
 }
 
 // Row-major C [M x N] = op(A) op(B) (+ bias, act = GELU(C)), or C += op(A)
@@ -410,7 +428,9 @@ int own_gemm(const char *op, hipStream_t st, bool ta, bool tb, int M, int N, int
 {
     if (!gpt_ops::gemm::fits(A, B, C, act, M, N, K, ta, tb))
         return 1;
-    gpt_ops::gemm::Choice c = own_choice(M, N, K, ta, tb);
+    OwnPlan spare;
+    OwnPlan *const plan = own_plan(M, N, K, ta, tb, &spare);
+    gpt_ops::gemm::Choice c = plan->c;
     // (rocBLAS, on the wide products, needs a pass of its own for the bias)
     float library_us = 7.f + 7.2e-9f * 2.f * M * N * K;
     if (!ta && library_us < 10.5f)
@@ -422,7 +442,10 @@ int own_gemm(const char *op, hipStream_t st, bool ta, bool tb, int M, int N, int
     int *ticket = nullptr;
     if (c.splits > 1 && !split_workspace(&part, &ticket, st))
         c = gpt_ops::gemm::choose(M, N, K, ta, tb, false);
-    return launched(op, gpt_ops::gemm::run(A, B, C, bias, act, M, N, K, ta, tb, add, c, part, ticket, st));
+    const int rc = launched(op, gpt_ops::gemm::run(A, B, C, bias, act, M, N, K, ta, tb, add, c, part, ticket, st));
+    if (rc == 0 && !plan->ran.exchange(true))
+        ++g_own_ran;
+    return rc;
 }
 
 // Row-major C = op(A) op(B), or C +=: this library's kernel, or hipBLASLt
@@ -789,16 +812,11 @@ int gpt_hip_ops_gemm_info(int *plans, int *tuned, int *blaslt_version)
     if (!plans || !tuned || !blaslt_version)
         return fail(GPT_HIP_OPS_ENULL, "gpt_hip_ops_gemm_info: NULL output");
     std::lock_guard<std::mutex> lock(g_lt_mu);
-    int np = 0, nt = 0;
+    int np = 0;
     for (int i = 0; i < g_nplans; ++i)
         np += g_plans[i].ok ? 1 : 0;
-    {
-        std::lock_guard<std::mutex> own(g_own_mu);
-        nt = g_nown;
-        np += nt;
-    }
-    *plans = np;
-    *tuned = nt;
+    *tuned = g_own_ran;
+    *plans = np + *tuned;
     *blaslt_version = 0;
     for (int d = 0; d < kMaxDevices; ++d)
         if (g_lt[d])

@@ -204,9 +204,9 @@ def device_fill_const(ptr, value, size, stream=None):
 
 
 def gemm_info() -> dict:
-    """{"plans", "tuned", "blaslt_version"}: the product shapes this process
-    has planned, how many of them run on the library's own kernel, and the
-    loaded hipBLASLt's version (0 before any hipBLASLt plan)."""
+    """{"plans", "tuned", "blaslt_version"}: the product shapes that have run on
+    the library's own kernels in this process ("tuned"), those and the hipBLASLt
+    plans made ("plans"), and the loaded hipBLASLt's version (0 before any plan)."""
     lib = load_library()
     vals = [ctypes.c_int(0) for _ in range(3)]
     rc = lib.gpt_hip_ops_gemm_info(*[ctypes.byref(v) for v in vals])

@@ -184,12 +184,12 @@ int gpt_hip_fill_const_f32(float *ptr, float value, size_t size, void *stream);
  * No reference counterpart (the reference prints and aborts). */
 const char *gpt_hip_ops_last_error(void);
 
-/* GEMM planning state, for tests and tuning: *plans = product shapes and
- * transposes planned so far in this process (and epilogues, on hipBLASLt),
- * *tuned = how many of them run on this library's own kernel with a launch
- * choice made for the shape, *blaslt_version = the loaded hipBLASLt's
- * hipblasLtGetVersion (0 before the first hipBLASLt plan). No reference
- * counterpart. */
+/* GEMM planning state, for tests and tuning: *tuned = product shapes and
+ * transposes that have run on this library's own kernels so far in this process
+ * (of the first 768 that they were considered for), *plans = those and the
+ * hipBLASLt plans made (one per shape, transposes and epilogue),
+ * *blaslt_version = the loaded hipBLASLt's hipblasLtGetVersion (0 before the
+ * first hipBLASLt plan). No reference counterpart. */
 int gpt_hip_ops_gemm_info(int *plans, int *tuned, int *blaslt_version);
 
 /* Frees the workspaces on the calling thread's current device after waiting

@@ -203,3 +203,48 @@ def test_errors_do_not_add_up_over_rows(dev, M, K, N, form):
     e = y.double() - x.double() @ w.double()
     alone = float(e.pow(2).mean().sqrt()) * M ** 0.5
     assert float(e.sum(0).pow(2).mean().sqrt()) < 1.3 * alone
+
+
+# (form, M, N, K, products on the library's own kernels). Per form a size for each tile
+# of ops_gemm.hip (128 x 128 .. 32 x 64, in its order), unsplit and with k split where
+# the rule does that, and one that the BLAS libraries take. "ta" is a whole linear
+# backward over K rows: grad_x and grad_w.
+ROUTES = [("nn", 2195, 2168, 40, 1), ("nn", 730, 2948, 656, 1), ("nn", 1637, 1180, 956, 1), ("nn", 568, 2872, 40, 1),
+          ("nn", 191, 2820, 352, 1), ("nn", 1059, 48, 60, 1), ("nn", 112, 2128, 1060, 1), ("nn", 577, 3252, 56, 1),
+          ("nn", 92, 3020, 1284, 1), ("nn", 3, 216, 88, 1), ("nn", 4, 40, 1032, 1), ("nn", 98, 2724, 40, 1),
+          ("nn", 79, 3172, 40, 1), ("nn", 700, 300, 1500, 0), ("nn", 77, 771, 768, 0),
+          ("nt", 2610, 1896, 36, 1), ("nt", 1584, 1524, 768, 1), ("nt", 624, 3204, 1420, 1), ("nt", 610, 2476, 36, 1),
+          ("nt", 126, 3488, 1680, 1), ("nt", 1221, 88, 48, 1), ("nt", 2314, 1708, 40, 1), ("nt", 4, 52, 100, 1),
+          ("nt", 1, 36, 700, 1), ("nt", 322, 864, 44, 1), ("nt", 147, 1664, 36, 1), ("nt", 700, 308, 1500, 0),
+          ("ta", 2164, 1252, 804, 2), ("ta", 636, 3264, 1875, 2), ("ta", 1504, 1048, 68, 2), ("ta", 1152, 1780, 748, 1),
+          ("ta", 52, 472, 60, 2), ("ta", 2708, 644, 116, 2), ("ta", 302, 406, 1000, 0)]
+
+
+@pytest.mark.parametrize("form,M,N,K,own", ROUTES)
+def test_which_products_the_own_kernels_take(dev, form, M, N, K, own):
+    """Sizes that no other test of the process calls, so that the count of shapes on the
+    own kernels tells where each product ran."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+
+    def rnd(*s):
+        return torch.empty(s, device=dev).normal_(0.0, 1.0, generator=g)
+
+    before = ops.gemm_info()
+    if form == "ta":
+        x, w, gy = rnd(K, M), rnd(M, N), rnd(K, N)
+        gx, gw, gb = torch.empty((K, M), device=dev), torch.zeros((M, N), device=dev), torch.zeros(N, device=dev)
+        ops.device_linear_backward(gx, gw, gb, gy, x, w, 1, K, M, N)
+        assert rel(gx, gy.double() @ w.double().t()) < tol(N)
+        assert rel(gw, x.double().t() @ gy.double()) < tol(K)
+    else:
+        x, w, b, y = rnd(M, K), rnd(K, N), torch.zeros(N, device=dev), torch.empty((M, N), device=dev)
+        if form == "nn":
+            ops.device_linear_activation_fused_forward(y, None, x, w, b, False, 1, M, K, N)
+        else:
+            ops.device_unembedding_forward(y, x, w.t().contiguous(), 1, M, K, N)
+        assert rel(y, x.double() @ w.double()) < tol(K)
+    after = ops.gemm_info()
+    assert after["tuned"] - before["tuned"] == own
+    assert after["plans"] - before["plans"] >= own

@@ -205,7 +205,7 @@ def test_linear_fwd_bwd(dev, B, T, n_in, n_out, activation):
                                                     (3072, 768, False)])
 def test_linear_at_gpt2_step_shapes(dev, n_in, n_out, activation):
     """The GPT-2 124M layer shapes at B=16, T=256 (4096 rows), where the
-    library takes its table of tuned GEMM kernels: y = x w + b, GELU, grad_x,
+    library's own tiled products are taken: y = x w + b, GELU, grad_x,
     grad_w (accumulated) and grad_b against float64 numpy (the oracle's C
     loops would take minutes here; its GELU, gelu_tanh in ops_oracle.c, is
     restated in float64)."""
@@ -233,19 +233,19 @@ def test_linear_at_gpt2_step_shapes(dev, n_in, n_out, activation):
     assert_close("linear grad_x", host(gx).reshape(-1, n_in), gy64 @ w64.T, RTOL)
     assert_close("linear grad_w", host(dgw), gw0.astype(np.float64) + x64.T @ gy64, RTOL)
     assert_close("linear grad_b", host(dgb), gb0.astype(np.float64) + gy64.sum(0), RTOL)
-    # the tuning table lists kernels of this (PyTorch-bundled) hipBLASLt for
-    # every one of these shapes: at least one plan must have taken one
+    # y, grad_x and grad_w of this layer have run on the own kernels by now (which
+    # of them did is counted in a process of its own, tests/torchfree_linear.py)
     info = ops.gemm_info()
     print("gemm plans:", info)
-    assert info["tuned"] >= 1, info
+    assert info["tuned"] >= 3, info
 
 
 def test_linear_at_gpt2_step_shapes_without_torch(dev):
     """The same four layer shapes in a process that never imports PyTorch
     (tests/torchfree_linear.py, device memory from the HIP runtime through
-    ctypes), where the library binds ROCm's own hipBLASLt, the build the
-    reference-side trainer and generator run on: parity against float64
-    numpy at 1e-5 and the tuned kernels taken."""
+    ctypes), where the library binds ROCm's own BLAS libraries, as in the
+    reference-side trainer and generator: parity against float64
+    numpy at 1e-5 and every product on the library's own kernels."""
     import subprocess
     import sys
 

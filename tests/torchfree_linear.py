@@ -1,12 +1,12 @@
 """The GPT-2 124M linear layers at the training step's 4096 rows through the
-ops library in a process that never imports PyTorch, so that the library
-binds ROCm's own hipBLASLt (the one the reference-side trainer and generator
-load), not the copy PyTorch bundles: the tuning table's kernels for that
-build are the ones exercised. Run by tests/test_ops_gpu.py in a subprocess;
+ops library in a process that never imports PyTorch, as the reference-side
+trainer and generator are (the library then binds ROCm's own BLAS libraries,
+not the copies PyTorch bundles). Run by tests/test_ops_gpu.py in a subprocess;
 device memory comes from the HIP runtime through ctypes. Checks y = x w + b
 (and GELU), grad_x, grad_w accumulated onto a nonzero start and grad_b
-against float64 numpy at 1e-5 norm-wise, and that the tuned kernels were
-taken. Exit status 0 on success."""
+against float64 numpy at 1e-5 norm-wise, and that all twelve products (four
+layers; y, grad_x and grad_w) ran on the library's own kernels. Exit status 0
+on success."""
 import ctypes
 import os
 import sys
@@ -86,7 +86,7 @@ def main():
     print("gemm plans:", info, "torch loaded:", "torch" in sys.modules, flush=True)
     assert "torch" not in sys.modules
     assert worst <= RTOL, worst
-    assert info["tuned"] >= 1, info
+    assert info["tuned"] == info["plans"] == 12, info
     return 0
 
 
