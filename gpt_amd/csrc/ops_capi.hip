@@ -111,19 +111,17 @@ int gemm_rm(const char *op, rocblas_handle h, bool ta, bool tb, int M, int N, in
 
 // ---------------------------------------------------------------- workspace
 
-// Workspaces, one buffer per (device, stream, purpose), kept until
+// Workspaces, one buffer per (device, stream) and purpose, kept until
 // gpt_hip_ops_release_workspaces or the process's end. Calls on one stream run
 // in order, so they can share its buffers; calls on different streams get
 // different ones. (A stream-ordered hipMallocAsync / hipFreeAsync pair per call
 // measured ~10 us of GPU time per call here, more than the reductions it
-// serves.) Slot 0: reduction partials (at most 256 partial rows, a few MB),
-// grown when a call needs more. Slot 1: a split product's tickets and partial
-// tiles (32 MB), never grown.
+// serves.) Reduction partials (at most 256 partial rows, a few MB) grow when a
+// call needs more; at most kMaxWorkspaces of them.
 struct Workspace
 {
     int dev;
     hipStream_t st;
-    int slot;
     float *p;
     size_t floats;
 };
@@ -132,28 +130,23 @@ std::mutex g_ws_mu;
 Workspace g_ws[kMaxWorkspaces];
 int g_ws_n = 0;
 
-// The entry of (current device, st, slot), made if there is room; g_ws_mu held.
-Workspace *ws_find(int dev, hipStream_t st, int slot)
-{
-    for (int i = 0; i < g_ws_n; ++i)
-        if (g_ws[i].dev == dev && g_ws[i].st == st && g_ws[i].slot == slot)
-            return &g_ws[i];
-    if (g_ws_n == kMaxWorkspaces)
-        return nullptr;
-    Workspace *w = &g_ws[g_ws_n++];
-    *w = Workspace{dev, st, slot, nullptr, 0};
-    return w;
-}
-
 int ws_get(const char *op, float **out, size_t floats, hipStream_t st)
 {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess)
         return fail(GPT_HIP_OPS_ENODEV, "%s: no current HIP device", op);
     std::lock_guard<std::mutex> lock(g_ws_mu);
-    Workspace *w = ws_find(dev, st, 0);
+    Workspace *w = nullptr;
+    for (int i = 0; i < g_ws_n; ++i)
+        if (g_ws[i].dev == dev && g_ws[i].st == st)
+            w = &g_ws[i];
     if (!w)
-        return fail(GPT_HIP_OPS_ENOMEM, "%s: more than %d (device, stream) workspaces", op, kMaxWorkspaces);
+    {
+        if (g_ws_n == kMaxWorkspaces)
+            return fail(GPT_HIP_OPS_ENOMEM, "%s: more than %d (device, stream) workspaces", op, kMaxWorkspaces);
+        w = &g_ws[g_ws_n++];
+        *w = Workspace{dev, st, nullptr, 0};
+    }
     if (w->floats < floats)
     {
         if (w->p)
@@ -176,13 +169,21 @@ int ws_get(const char *op, float **out, size_t floats, hipStream_t st)
     return 0;
 }
 
+// A split product's tickets and partial tiles, 32 MB that never grow. At most
+// kMaxSplit streams of a device hold one, in a table of their own.
+struct SplitWorkspace
+{
+    hipStream_t st;
+    float *p;
+};
+constexpr int kMaxSplit = 16;
+SplitWorkspace g_split[kMaxDevices][kMaxSplit];  // (g_ws_mu); p = null: free
+
 // Tickets and partial tiles for a split product on `st`; false where there are
 // none to be had (then the product runs unsplit): while the stream is captured,
 // since a graph may be replayed on any stream, beside eager calls on this one;
 // on hipStreamPerThread, whose handle names a stream of each thread; or when
-// memory or table entries have run out. At most kMaxSplit streams hold
-// one, so that the reduction partials keep table entries to themselves.
-constexpr int kMaxSplit = 16;
+// memory or table entries have run out.
 bool split_workspace(float **part, int **ticket, hipStream_t st)
 {
     using namespace gpt_ops::gemm;
@@ -193,22 +194,23 @@ bool split_workspace(float **part, int **ticket, hipStream_t st)
         return false;
     }
     int dev = 0;
-    if (cs != hipStreamCaptureStatusNone || st == hipStreamPerThread || hipGetDevice(&dev) != hipSuccess)
+    if (cs != hipStreamCaptureStatusNone || st == hipStreamPerThread || hipGetDevice(&dev) != hipSuccess || dev < 0 ||
+        dev >= kMaxDevices)
         return false;
     std::lock_guard<std::mutex> lock(g_ws_mu);
-    int held = 0;
-    Workspace *w = nullptr;
-    for (int i = 0; i < g_ws_n; ++i)
+    SplitWorkspace *w = nullptr, *free = nullptr;
+    for (SplitWorkspace &e : g_split[dev])
     {
-        held += g_ws[i].slot == 1;
-        if (g_ws[i].dev == dev && g_ws[i].st == st && g_ws[i].slot == 1)
-            w = &g_ws[i];
+        if (e.p && e.st == st)
+            w = &e;
+        if (!e.p && !free)
+            free = &e;
     }
-    if (!w && (held >= kMaxSplit || !(w = ws_find(dev, st, 1))))
-        return false;
-    if (!w->p)
+    if (!w)
     {
         void *q = nullptr;
+        if (!free)
+            return false;
         if (hipMalloc(&q, (kMaxTickets + kPartFloats) * sizeof(float)) != hipSuccess)
         {
             (void)hipGetLastError();
@@ -219,8 +221,8 @@ bool split_workspace(float **part, int **ticket, hipStream_t st)
             (void)hipFree(q);
             return false;
         }
-        w->p = static_cast<float *>(q);
-        w->floats = kMaxTickets + kPartFloats;
+        w = free;
+        *w = SplitWorkspace{st, static_cast<float *>(q)};
     }
     *ticket = reinterpret_cast<int *>(w->p);
     *part = w->p + kMaxTickets;
@@ -850,6 +852,12 @@ int gpt_hip_ops_release_workspaces(void)
             g_ws[keep++] = g_ws[i];
     }
     g_ws_n = keep;
+    if (dev >= 0 && dev < kMaxDevices)
+        for (SplitWorkspace &w : g_split[dev])
+        {
+            (void)hipFree(w.p);
+            w = SplitWorkspace{};
+        }
     return 0;
 }
 
