@@ -169,60 +169,97 @@ int ws_get(const char *op, float **out, size_t floats, hipStream_t st)
     return 0;
 }
 
-// A split product's tickets and partial tiles, 32 MB that never grow. At most
-// kMaxSplit streams of a device hold one, in a table of their own.
+// A split product's tickets and partial tiles, 32 MB that never grow, for the
+// eager calls of a stream or for one capture on it. A graph has one of its own,
+// since it may be replayed on any stream, beside eager calls on the one that it
+// was captured on, and keeps it: nothing tells when it is destroyed. At most
+// kMaxSplit of either kind on a device, in a table of their own.
 struct SplitWorkspace
 {
     hipStream_t st;
+    unsigned long long capture;
     float *p;
 };
 constexpr int kMaxSplit = 16;
-SplitWorkspace g_split[kMaxDevices][kMaxSplit];  // (g_ws_mu); p = null: free
+SplitWorkspace g_split[2][kMaxDevices][kMaxSplit];  // [captured] (g_ws_mu); p = null: free
+
+// hipMalloc is refused, and ends the capture, while any stream is captured in
+// the default mode, but for a thread in this one.
+struct RelaxedCapture
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// A new one, its tickets cleared on *st, or where st is null (a captured stream,
+// whose graph would clear them again on every replay, 5 us) by work that has
+// ended. Null where there is no memory.
+float *new_split_workspace(const hipStream_t *st)
+{
+    const RelaxedCapture relaxed;
+    void *q = nullptr;
+    hipError_t e = hipMalloc(&q, (gpt_ops::gemm::kMaxTickets + gpt_ops::gemm::kPartFloats) * sizeof(float));
+    if (e != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    hipStream_t own = nullptr;
+    if (!st)
+        e = hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
+    if (e == hipSuccess)
+        e = gpt_ops::launch_fill_const(static_cast<float *>(q), gpt_ops::gemm::kMaxTickets, 0.f, st ? *st : own);
+    if (own)
+    {
+        const hipError_t sync = hipStreamSynchronize(own);
+        e = e == hipSuccess ? sync : e;
+        (void)hipStreamDestroy(own);
+    }
+    if (e == hipSuccess)
+        return static_cast<float *>(q);
+    (void)hipGetLastError();
+    (void)hipFree(q);
+    return nullptr;
+}
 
 // Tickets and partial tiles for a split product on `st`; false where there are
-// none to be had (then the product runs unsplit): while the stream is captured,
-// since a graph may be replayed on any stream, beside eager calls on this one;
-// on hipStreamPerThread, whose handle names a stream of each thread; or when
-// memory or table entries have run out.
-bool split_workspace(float **part, int **ticket, hipStream_t st)
+// none to be had: on hipStreamPerThread, whose handle names a stream of each
+// thread, or when memory or table entries have run out. *capturing: whether the
+// stream is being captured.
+bool split_workspace(float **part, int **ticket, bool *capturing, hipStream_t st)
 {
     using namespace gpt_ops::gemm;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cs) != hipSuccess)
+    unsigned long long id = 0;
+    *capturing = true;
+    if (hipStreamGetCaptureInfo(st, &cs, &id) != hipSuccess)
     {
         (void)hipGetLastError();
         return false;
     }
+    *capturing = cs != hipStreamCaptureStatusNone;
     int dev = 0;
-    if (cs != hipStreamCaptureStatusNone || st == hipStreamPerThread || hipGetDevice(&dev) != hipSuccess || dev < 0 ||
-        dev >= kMaxDevices)
+    if ((!*capturing && st == hipStreamPerThread) || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
         return false;
     std::lock_guard<std::mutex> lock(g_ws_mu);
     SplitWorkspace *w = nullptr, *free = nullptr;
-    for (SplitWorkspace &e : g_split[dev])
+    for (SplitWorkspace &e : g_split[*capturing][dev])
     {
-        if (e.p && e.st == st)
+        if (e.p && e.st == st && (!*capturing || e.capture == id))
             w = &e;
         if (!e.p && !free)
             free = &e;
     }
     if (!w)
     {
-        void *q = nullptr;
         if (!free)
             return false;
-        if (hipMalloc(&q, (kMaxTickets + kPartFloats) * sizeof(float)) != hipSuccess)
-        {
-            (void)hipGetLastError();
+        float *const q = new_split_workspace(*capturing ? nullptr : &st);
+        if (!q)
             return false;
-        }
-        if (gpt_ops::launch_fill_const(static_cast<float *>(q), kMaxTickets, 0.f, st) != hipSuccess)
-        {
-            (void)hipFree(q);
-            return false;
-        }
         w = free;
-        *w = SplitWorkspace{st, static_cast<float *>(q)};
+        *w = SplitWorkspace{st, id, q};
     }
     *ticket = reinterpret_cast<int *>(w->p);
     *part = w->p + kMaxTickets;
@@ -252,7 +289,8 @@ bool split_workspace(float **part, int **ticket, hipStream_t st)
 // per shape, so results are bitwise reproducible. One hipBLASLt plan
 // (descriptor, layouts, heuristic algorithm) per (device, shape, transposes,
 // epilogue), built on first use and kept; rocBLAS takes any shape hipBLASLt has
-// no plan for.
+// no plan for. (A product that splits k takes another kernel, and with it other
+// bits, where it gets no split workspace.)
 struct LtPlan
 {
     int dev;
@@ -390,7 +428,7 @@ struct OwnPlan
     int M, N, K;
     bool ta, tb;
     std::atomic<bool> ran;
-    gpt_ops::gemm::Choice c;
+    gpt_ops::gemm::Choice c, plain;  // plain: the best without a split
 };
 constexpr int kOwnPlans = 1024, kOwnFull = 768;
 std::mutex g_own_mu;
@@ -419,7 +457,24 @@ OwnPlan *own_plan(int M, int N, int K, bool ta, bool tb, OwnPlan *spare)
     p->M = M, p->N = N, p->K = K, p->ta = ta, p->tb = tb;
     p->ran = p == spare;
     p->c = gpt_ops::gemm::choose(M, N, K, ta, tb, true);
+    p->plain = p->c.splits > 1 ? gpt_ops::gemm::choose(M, N, K, ta, tb, false) : p->c;
     return p;
+}
+
+// Whether the handle is there that a product on the libraries takes: they cannot
+// make one while a stream is captured.
+bool library_ready(bool ta, int N)
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+        return false;
+    if (use_lt(ta, N))
+    {
+        std::lock_guard<std::mutex> lock(g_lt_mu);
+        return g_lt[dev];
+    }
+    std::lock_guard<std::mutex> lock(g_blas_mu);
+    return g_blas[dev];
 }
 
 // Row-major C [M x N] = op(A) op(B) (+ bias, act = GELU(C)), or C += op(A)
@@ -438,12 +493,20 @@ int own_gemm(const char *op, hipStream_t st, bool ta, bool tb, int M, int N, int
     if (!ta && library_us < 10.5f)
         library_us = 10.5f;
     library_us += bias && !use_lt(ta, N) ? 3.f : 0.f;
-    if (c.us > library_us * (ta ? 0.95f : M <= 128 ? 1.3f : 1.f))
+    const float limit_us = library_us * (ta ? 0.95f : M <= 128 ? 1.3f : 1.f);
+    if (c.us > limit_us)
         return 1;
     float *part = nullptr;
     int *ticket = nullptr;
-    if (c.splits > 1 && !split_workspace(&part, &ticket, st))
-        c = gpt_ops::gemm::choose(M, N, K, ta, tb, false);
+    bool capturing = false;
+    if (c.splits > 1 && !split_workspace(&part, &ticket, &capturing, st))
+    {
+        // unsplit, unless the libraries are faster then (x^T grad_y of 768 x 768
+        // over 4096 rows: 125 us against 42)
+        c = plan->plain;
+        if (c.us > limit_us && (!capturing || library_ready(ta, N)))
+            return 1;
+    }
     const int rc = launched(op, gpt_ops::gemm::run(A, B, C, bias, act, M, N, K, ta, tb, add, c, part, ticket, st));
     if (rc == 0 && !plan->ran.exchange(true))
         ++g_own_ran;
@@ -853,7 +916,7 @@ int gpt_hip_ops_release_workspaces(void)
     }
     g_ws_n = keep;
     if (dev >= 0 && dev < kMaxDevices)
-        for (SplitWorkspace &w : g_split[dev])
+        for (SplitWorkspace &w : g_split[0][dev])  // (a graph's may be replayed yet)
         {
             (void)hipFree(w.p);
             w = SplitWorkspace{};

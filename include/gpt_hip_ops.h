@@ -33,10 +33,13 @@
  *     own HIP kernels. Reductions that need partial sums (LayerNorm and bias
  *     gradients, the gradient norm) use a workspace the library allocates on
  *     first use, one per (device, stream), grown when a call needs more (at
- *     most 256 partial rows: a few MB); products whose k range is split over
- *     workgroups use another of 32 MB (not under stream capture or on
- *     hipStreamPerThread, where they run unsplit and need none). Both are kept until
- *     gpt_hip_ops_release_workspaces or the process's end.
+ *     most 256 partial rows: a few MB; at most 64). Products whose k range is
+ *     split over workgroups use another of 32 MB: up to 16 streams of a device
+ *     hold one, and up to 16 graphs captured there (one per stream of the capture).
+ *     Where none is to be had (past those, on hipStreamPerThread, out of memory)
+ *     such a product runs unsplit or on the BLAS libraries, to the same precision
+ *     but other bits. Workspaces are kept until gpt_hip_ops_release_workspaces or
+ *     the process's end, a captured graph's until the process's end.
  *   - Token ids must lie in [0, vocab_rows) where the entry point takes
  *     vocab_rows > 0; the reference's methods do not receive the vocabulary
  *     size and do not check, and vocab_rows = 0 keeps that behaviour.

@@ -124,9 +124,8 @@ def test_second_pass_where_few_lanes_overflow(dev, row, col):
 
 
 def test_captured_products_replay(dev):
-    """A captured linear layer (which takes no split-k workspace) replayed
-    between eager calls gives the eager results' values, and the same bits on
-    every replay."""
+    """A captured linear layer replayed between eager calls gives the eager
+    results' values, and the same bits on every replay."""
     import torch
 
     M, K, N = 4096, 3072, 768

@@ -1,6 +1,8 @@
 """The ops library's workspaces: as many streams as its table of reduction
 buffers has entries, each with products that split k as well, through a linear
-layer's backward (products, bias gradient) against float64."""
+layer's backward (products, bias gradient) against float64; captured products
+that split k, which are the eager ones bit for bit, and more captures than hold a
+split workspace."""
 import ctypes
 
 import pytest
@@ -55,3 +57,93 @@ def test_backward_on_64_streams(dev, streams):
     rx, rw, rb = gy.double() @ w.double().t(), x.double().t() @ gy.double(), gy.double().sum(0)
     for i in range(STREAMS):
         assert rel(gx[i], rx) < 1.2e-6 and rel(gw[i], rw) < 3e-7 and rel(gb[i], rb) < 3e-7, i
+
+
+def captured(fn):
+    import torch
+
+    st, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.graph(graph, stream=st):
+        fn(st)
+    return graph, st
+
+
+@pytest.mark.parametrize("M,K,N", [(77, 768, 3072), (4096, 768, 768)])
+def test_captured_split_products_are_the_eager_ones(dev, M, K, N):
+    """grad_y w^T splits k at the first size, x^T grad_y at the second. The graph is
+    replayed on a stream of its own while eager calls run on the one it was captured
+    on; both give the eager bits each time."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(M)
+    x, w, gy = (torch.empty(s, device=dev).normal_(0.0, 1.0, generator=g) for s in ((M, K), (K, N), (M, N)))
+    out = [[torch.zeros(s, device=dev) for s in ((M, K), (K, N), (N,))] for _ in range(3)]
+
+    def backward(o, st):
+        ops.device_linear_backward(*o, gy, x, w, 1, M, K, N, stream=st)
+
+    first = torch.cuda.Stream()
+    first.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(first):
+        backward(out[0], first)
+        first.synchronize()
+        graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=first):
+        backward(out[1], first)
+    other = torch.cuda.Stream()
+    for _ in range(4):
+        for o in out[1:]:
+            o[1].zero_(), o[2].zero_(), o[0].fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graph.replay()
+        backward(out[2], first)
+        torch.cuda.synchronize()
+        # (grad_b's reduction shares its buffer with the capture's stream, and is not compared)
+        for o in out[1:]:
+            assert torch.equal(o[0], out[0][0]) and torch.equal(o[1], out[0][1])
+
+
+def test_first_split_product_of_a_stream_beside_a_capture(dev):
+    """An eager product that allocates its split workspace while another stream is
+    being captured ends neither."""
+    import torch
+
+    M, K, N = 77, 3072, 768
+    g = torch.Generator(device=dev).manual_seed(6)
+    x, w = (torch.empty(s, device=dev).normal_(0.0, 1.0, generator=g) for s in ((M, K), (K, N)))
+    b, y, z = torch.zeros(N, device=dev), torch.empty((M, N), device=dev), torch.zeros(4, device=dev)
+    eager = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    ops.release_workspaces()
+
+    def both(st):
+        z.add_(1.0)
+        ops.device_linear_activation_fused_forward(y, None, x, w, b, False, 1, M, K, N, stream=eager)
+
+    graph, _ = captured(both)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert z.tolist() == [1.0] * 4
+    assert rel(y, x.double() @ w.double()) < 1.2e-6
+
+
+def test_more_captures_than_split_workspaces(dev):
+    import torch
+
+    M, K, N = 77, 3072, 768
+    g = torch.Generator(device=dev).manual_seed(5)
+    x, w = (torch.empty(s, device=dev).normal_(0.0, 1.0, generator=g) for s in ((M, K), (K, N)))
+    b, r = torch.zeros(N, device=dev), x.double() @ w.double()
+    made = []
+    for _ in range(20):
+        y = torch.full((M, N), float("nan"), device=dev)
+        made.append((captured(lambda st: ops.device_linear_activation_fused_forward(y, None, x, w, b, False, 1, M, K, N,
+                                                                                      stream=st)), y))
+    for _ in range(2):
+        for (graph, _), y in made:
+            y.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert rel(y, r) < 1.2e-6
