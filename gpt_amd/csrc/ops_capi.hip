@@ -111,19 +111,31 @@ int gemm_rm(const char *op, rocblas_handle h, bool ta, bool tb, int M, int N, in
 
 // ---------------------------------------------------------------- workspace
 
+// hipMalloc is refused, and ends the capture, while any stream is captured in
+// the default mode, but for a thread in this one.
+struct RelaxedCapture
+{
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // Workspaces, one buffer per (device, stream) and purpose, kept until
 // gpt_hip_ops_release_workspaces or the process's end. Calls on one stream run
 // in order, so they can share its buffers; calls on different streams get
 // different ones. (A stream-ordered hipMallocAsync / hipFreeAsync pair per call
 // measured ~10 us of GPU time per call here, more than the reductions it
 // serves.) Reduction partials (at most 256 partial rows, a few MB) grow when a
-// call needs more; at most kMaxWorkspaces of them.
+// call needs more; at most kMaxWorkspaces of them. A graph holds the address that
+// its calls were captured with: a buffer that a capture got is not freed any more
+// (nothing tells when the graph is destroyed).
 struct Workspace
 {
     int dev;
     hipStream_t st;
     float *p;
     size_t floats;
+    bool captured;
 };
 constexpr int kMaxWorkspaces = 64;
 std::mutex g_ws_mu;
@@ -145,18 +157,31 @@ int ws_get(const char *op, float **out, size_t floats, hipStream_t st)
         if (g_ws_n == kMaxWorkspaces)
             return fail(GPT_HIP_OPS_ENOMEM, "%s: more than %d (device, stream) workspaces", op, kMaxWorkspaces);
         w = &g_ws[g_ws_n++];
-        *w = Workspace{dev, st, nullptr, 0};
+        *w = Workspace{dev, st, nullptr, 0, false};
     }
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess)
+        (void)hipGetLastError();
+    const bool capturing = cs != hipStreamCaptureStatusNone;
     if (w->floats < floats)
     {
-        if (w->p)
+        const RelaxedCapture relaxed;
+        if (w->p && (w->captured || capturing))
+        {
+            // left to the graph, or to work queued before a capture that cannot
+            // wait for it; at least twice the size takes its place, so that all
+            // that are left come to less than the last
+            floats = floats > 2 * w->floats ? floats : 2 * w->floats;
+        }
+        else if (w->p)
         {
             // the old buffer may still be read by work queued on this stream
             if (hipStreamSynchronize(st) != hipSuccess || hipFree(w->p) != hipSuccess)
                 return fail(GPT_HIP_OPS_ELAUNCH, "%s: workspace release failed", op);
-            w->p = nullptr;
-            w->floats = 0;
         }
+        w->p = nullptr;
+        w->floats = 0;
+        w->captured = false;
         void *q = nullptr;
         const hipError_t e = hipMalloc(&q, floats * sizeof(float));
         if (e != hipSuccess)
@@ -165,6 +190,7 @@ int ws_get(const char *op, float **out, size_t floats, hipStream_t st)
         w->p = static_cast<float *>(q);
         w->floats = floats;
     }
+    w->captured |= capturing;
     *out = w->p;
     return 0;
 }
@@ -182,15 +208,6 @@ struct SplitWorkspace
 };
 constexpr int kMaxSplit = 16;
 SplitWorkspace g_split[2][kMaxDevices][kMaxSplit];  // [captured] (g_ws_mu); p = null: free
-
-// hipMalloc is refused, and ends the capture, while any stream is captured in
-// the default mode, but for a thread in this one.
-struct RelaxedCapture
-{
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
-};
 
 // A new one, its tickets cleared on *st, or where st is null (a captured stream,
 // whose graph would clear them again on every replay, 5 us) by work that has
@@ -909,7 +926,7 @@ int gpt_hip_ops_release_workspaces(void)
     int keep = 0;
     for (int i = 0; i < g_ws_n; ++i)
     {
-        if (g_ws[i].dev == dev)
+        if (g_ws[i].dev == dev && !g_ws[i].captured)
             (void)hipFree(g_ws[i].p);
         else
             g_ws[keep++] = g_ws[i];

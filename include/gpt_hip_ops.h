@@ -39,7 +39,9 @@
  *     Where none is to be had (past those, on hipStreamPerThread, out of memory)
  *     such a product runs unsplit or on the BLAS libraries, to the same precision
  *     but other bits. Workspaces are kept until gpt_hip_ops_release_workspaces or
- *     the process's end, a captured graph's until the process's end.
+ *     the process's end, those that a captured call got until the process's end. A
+ *     graph's reductions share the buffer of the stream that it was captured on:
+ *     its replays must not overlap work on that stream that needs it too.
  *   - Token ids must lie in [0, vocab_rows) where the entry point takes
  *     vocab_rows > 0; the reference's methods do not receive the vocabulary
  *     size and do not check, and vocab_rows = 0 keeps that behaviour.
@@ -197,7 +199,8 @@ int gpt_hip_ops_gemm_info(int *plans, int *tuned, int *blaslt_version);
 
 /* Frees the workspaces on the calling thread's current device after waiting
  * for all work queued there; the next call that needs one allocates again.
- * Calls on other host threads must not overlap it. Returns 0, or
+ * Those that calls under stream capture were given stay, for the graphs that hold
+ * their addresses. Calls on other host threads must not overlap it. Returns 0, or
  * GPT_HIP_OPS_ENODEV / GPT_HIP_OPS_ELAUNCH. No reference counterpart. */
 int gpt_hip_ops_release_workspaces(void);
 

@@ -129,6 +129,64 @@ def test_first_split_product_of_a_stream_beside_a_capture(dev):
     assert rel(y, x.double() @ w.double()) < 1.2e-6
 
 
+def test_graphs_outlive_a_release_and_a_larger_call(dev):
+    """A captured LayerNorm backward, linear backward and clipping call keep the
+    buffer that they were captured with when the workspaces are released, and when a
+    larger call on the stream needs more; memory allocated afterwards is not theirs."""
+    import torch
+
+    M, C = 512, 768
+    g = torch.Generator(device=dev).manual_seed(9)
+
+    def rnd(*s):
+        return torch.empty(s, device=dev).normal_(0.0, 1.0, generator=g)
+
+    x, w, gy, gamma = rnd(M, C), rnd(C, C), rnd(M, C), rnd(C)
+    mean, var = x.mean(1), x.var(1, unbiased=False)
+    big = rnd(4096, 4 * C), rnd(4096, C), rnd(C, 4 * C)
+    big_out = torch.empty((4096, C), device=dev), torch.zeros((C, 4 * C), device=dev), torch.zeros(4 * C, device=dev)
+    out = [torch.zeros(s, device=dev) for s in ((M, C), (C,), (C,), (M, C), (C, C), (C,))]
+    clip = gy.clone()
+
+    def calls(st):
+        ops.device_layernorm_residual_fused_backward(*out[:3], gy, None, x, mean, var, gamma, 1, M, C, stream=st)
+        ops.device_linear_backward(*out[3:], gy, x, w, 1, M, C, C, stream=st)
+        ops.device_scale_and_clip_grad(clip, M * C, 1.0, 1, stream=st)
+
+    def reset():
+        for o in out:
+            o.zero_()
+        clip.copy_(gy)
+        torch.cuda.synchronize()
+
+    torch.cuda.synchronize()
+    ops.release_workspaces()
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    calls(st)
+    torch.cuda.synchronize()
+    want = [t.clone() for t in out + [clip]]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        calls(st)
+    for step in range(4):
+        if step == 1:
+            ops.release_workspaces()
+        if step == 2:
+            ops.device_linear_backward(*big_out, big[0], big[1], big[2], 1, 4096, C, 4 * C, stream=st)
+            torch.cuda.synchronize()
+        if step == 3:
+            ops.release_workspaces()
+        held = [torch.full((1 << 18,), 7.0, device=dev) for _ in range(64)]  # 64 MB of what might have been freed
+        reset()
+        graph.replay()
+        torch.cuda.synchronize()
+        for t, e in zip(out + [clip], want):
+            assert torch.equal(t, e), step
+        assert all(bool((h == 7.0).all()) for h in held), step
+        del held
+
+
 def test_more_captures_than_split_workspaces(dev):
     import torch
 
