@@ -953,7 +953,7 @@ __global__ __launch_bounds__(256) void adamw_kernel(float *__restrict__ p, const
     }
 }
 
-constexpr int kClipParts = 1024;
+constexpr int kClipParts = 1024, kClipPartsMost = 4096;
 
 // Partial sums of (g / accum)^2 over fixed stripes: workgroup p covers
 // elements [p * stripe, (p + 1) * stripe) (stripe a multiple of 4); g is not
@@ -961,7 +961,10 @@ constexpr int kClipParts = 1024;
 // the scaled values; the same scaled values are formed here and again when
 // they are written). 1024 stripes (every workgroup of the second pass adds
 // them all up again), eight float4 in flight per thread; no division where
-// accum is 1, which is exact: 124 M elements 132 -> 85 us, 5.8 TB/s.
+// accum is 1, which is exact: 124 M elements 132 -> 85 us, 5.8 TB/s. The scalar
+// form, with one load in flight per thread, takes 4096 stripes from 16 Mi elements
+// on (both passes, accum 2: 124 M + 1 elements 420 us, 509 with 1024; 20 M + 3 57
+// and 61; but 5 M + 1 31 and 27).
 template <bool V4>
 __global__ __launch_bounds__(256) void clip_partial_kernel(float *__restrict__ part, const float *__restrict__ g,
                                                            long n, long stripe, float accum)
@@ -1298,26 +1301,27 @@ hipError_t launch_adamw(float *p, const float *g, float *m, float *v, long n, fl
     return hipGetLastError();
 }
 
-int clip_parts() { return kClipParts; }
+int clip_parts() { return kClipPartsMost; }
 
 hipError_t launch_scale_clip(float *g, long n, float max_norm, float accum, float *ws, hipStream_t st)
 {
     const bool v4 = n % 4 == 0 && al16(g);
-    long stripe = (n + kClipParts - 1) / kClipParts;
+    const int parts = v4 || n < 1L << 24 ? kClipParts : kClipPartsMost;
+    long stripe = (n + parts - 1) / parts;
     stripe = (stripe + 3) & ~3L;
     if (v4)
-        hipLaunchKernelGGL(clip_partial_kernel<true>, dim3(kClipParts), dim3(256), 0, st, ws, g, n, stripe, accum);
+        hipLaunchKernelGGL(clip_partial_kernel<true>, dim3(parts), dim3(256), 0, st, ws, g, n, stripe, accum);
     else
-        hipLaunchKernelGGL(clip_partial_kernel<false>, dim3(kClipParts), dim3(256), 0, st, ws, g, n, stripe, accum);
+        hipLaunchKernelGGL(clip_partial_kernel<false>, dim3(parts), dim3(256), 0, st, ws, g, n, stripe, accum);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
     if (v4)
         hipLaunchKernelGGL(clip_apply_kernel<true>, dim3(grid_for(n / 4, 256, 8192)), dim3(256), 0, st, g, ws,
-                           kClipParts, n, max_norm, accum);
+                           parts, n, max_norm, accum);
     else
         hipLaunchKernelGGL(clip_apply_kernel<false>, dim3(grid_for(n, 256, 8192)), dim3(256), 0, st, g, ws,
-                           kClipParts, n, max_norm, accum);
+                           parts, n, max_norm, accum);
     return hipGetLastError();
 }
 

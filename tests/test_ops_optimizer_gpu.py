@@ -29,7 +29,7 @@ def test_adamw_sizes(dev, n):
         assert np.all(t[n:] == 7)
 
 
-@pytest.mark.parametrize("n", [3, 4096, 1024 * 1024 + 4, 9000001])
+@pytest.mark.parametrize("n", [3, 4096, 1024 * 1024 + 4, 9000001, (1 << 24) + 1])
 @pytest.mark.parametrize("max_norm,accum", [(1e9, 1), (0.5, 1), (1e9, 3), (0.5, 3)])
 def test_clip(dev, n, max_norm, accum):
     import torch
