@@ -288,17 +288,22 @@ bool split_workspace(float **part, int **ticket, bool *capturing, hipStream_t st
 // The library's own kernels (ops_gemm.hip) take every product whose rows are
 // 16-byte aligned multiples of 4 floats and that they finish first by their
 // time model, against 7 us plus 7.2 us per GFLOP, but 10.5 us at least except for
-// weight gradients, for the BLAS libraries (150 x 768 x 768: 11.2 us, here 8.7;
-// their fp32 kernels at 77 .. 1024 rows: 10.5-12 us up to 0.6 GFLOP, 27-30 at
-// 2.4, 40-43 at 4.8). The libraries' fp32 kernels stay ahead between the sizes of
-// gemm_rows_kernel and those that fill the card with tiles: 512 rows of 768 x
-// 768 10.8 against 17 us, 1024 rows of 3072 x 768 40 against 44 (1024 of 768 x
-// 3072: 43 against 36 us, 4096: 152 against 110). The model is of operands in
-// cache. Weights that come from memory, as while generating, cost the libraries
-// more (77 rows, GPT-2's four linear layers: 57 us and 8 for bias and GELU
-// passes, against 50), so up to 128 rows this library's kernel may be modelled
-// 1.3 times slower; weight gradients of few rows are modelled low, so there it
-// has to be 0.95 times.
+// weight gradients, for the BLAS libraries. The 10.5 us are the libraries' host
+// time: a call takes 12 us on the host, here 5 to 6, and the first one of every new
+// row count, as each step of generating makes them, 212 us on hipBLASLt for its
+// plan. In a captured graph, where that time is paid once, small products are
+// faster on the libraries (77 x 768 x 768: the kernels alone 6 us, here 8.6).
+// With the host time counted, over 224 sizes of each form from 1 to 4096 rows, the
+// rule's choices take 0.73 (forward), 0.81 (grad_y w^T) and 0.89 (x^T grad_y) of
+// the libraries' time in the geometric mean, and are more than 8 % slower in 14, 10
+// and 23 of them: mostly between the sizes of gemm_rows_kernel and those that fill
+// the card with tiles (384 x 768 x 2304 31 against 19 us, 1024 rows of 3072 x 768
+// 53 against 43, x^T grad_y of 1024 x 1024 over 1536 rows 47 against 29). At 4096
+// rows: 768 x 3072 110 against 152 us. The model is of operands in cache.
+// Weights that come from memory, as while generating, cost the libraries more (77
+// rows, GPT-2's four linear layers: 57 us and 8 for bias and GELU passes, against
+// 50), so up to 128 rows this library's kernel may be modelled 1.3 times slower;
+// weight gradients of few rows are modelled low, so there it has to be 0.95 times.
 // Between the two libraries a fixed rule decides (use_lt): hipBLASLt's fp32
 // kernels win where the row-major product has at most 1024 columns and for the
 // weight gradients x^T grad_y, and fuse the linear layer's bias (and GELU) into
