@@ -1,6 +1,6 @@
-// Element-wise device functions shared by the ops library's kernels. Written in
-// the reference CPU backend's operation order; the library is compiled without
-// FMA contraction.
+// Element-wise device functions shared by the ops library's kernels: the reference
+// CPU backend's GELU, in forms that lose less. The library is compiled without
+// FMA contraction; what is fused is written so.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -10,30 +10,40 @@
 
 namespace gpt_ops {
 
-constexpr float kGeluC = 0.79788456f;  // sqrt(2/pi) as the reference writes it (cpu_backend.cpp:234)
-constexpr float kGeluA = 0.044715f;
-constexpr float kGeluD = 0.107032f;  // 3 * 0.044715 * sqrt(2/pi) (cpu_backend.cpp:281)
+// GELU in its tanh form, 0.5 x (1 + tanh u), u = sqrt(2/pi) (x + 0.044715 x^3) with
+// the constants as the reference writes them (cpu_backend.cpp:234, :281). With
+// e = exp(-2|u|) and r = e / (1 + e) it is x - x r where x >= 0 and x r elsewhere,
+// and its derivative 1 - r or r, plus 2 x r / (1 + e) u': no 1 + tanh or 1 - tanh^2
+// whose cancellation would be left, and r, at most a half, is all that carries the
+// rounding of exp. Against 64 bits, N(0, 3): 2-norm 2.1e-8 (x / (1 + exp(-2u)):
+// 3.5e-8, 0.5 x (1 + tanh u): 2.8e-8), the derivative 3.6e-8 (3.6e-7, 1.4e-7).
+constexpr float kGeluE = -2.88539008f * 0.79788456f;  // -2 log2(e) sqrt(2/pi)
+constexpr float kGeluE3 = kGeluE * 0.044715f;
+constexpr float kGeluD = 2.0f * 0.79788456f;
+constexpr float kGeluD3 = 2.0f * 0.107032f;  // 2 * 3 * 0.044715 * sqrt(2/pi)
 
-// GELU in its tanh form, 0.5 s (1 + tanh u), as s / (1 + exp(-2u)): the same
-// function without the cancellation of 1 + tanh, in a third of tanhf's
-// instructions. exp(-2u) past the largest float gives s / inf = 0, the limit.
-__device__ __forceinline__ float gelu_sigmoid(float x)
+// r and 1 / (1 + e); past the largest float of x^3, e = 0.
+__device__ __forceinline__ float gelu_rest(float x, float *q)
 {
-    const float u = kGeluC * (x + kGeluA * x * x * x);
-    return 1.0f / (1.0f + __builtin_amdgcn_exp2f(-2.88539008f * u));  // 2 log2(e)
+    const float e = __builtin_amdgcn_exp2f(-fabsf(x * fmaf(kGeluE3, x * x, kGeluE)));
+    *q = 1.0f / (1.0f + e);
+    return e * *q;
 }
 
-__device__ __forceinline__ float gelu(float s)
+__device__ __forceinline__ float gelu(float x)
 {
-    return s * gelu_sigmoid(s);
+    float q;
+    const float r = gelu_rest(x, &q);
+    // (infinity keeps its value: -FLT_MAX * 0 + inf)
+    return x >= 0.0f ? fmaf(-fminf(x, 3.40282347e38f), r, x) : x * r;
 }
 
-// Its derivative, 0.5 (1 + tanh u) + 0.5 x (1 - tanh^2 u) u', with tanh u =
-// 2 g - 1.
 __device__ __forceinline__ float gelu_grad(float x)
 {
-    const float g = gelu_sigmoid(x);
-    return g + 2.0f * x * g * (1.0f - g) * (kGeluC + kGeluD * x * x);
+    float q;
+    const float r = gelu_rest(x, &q);
+    const float s = fmaf(x * (r * q), fmaf(kGeluD3, x * x, kGeluD), x >= 0.0f ? -r : r);
+    return x >= 0.0f ? 1.0f + s : s;
 }
 
 }  // namespace gpt_ops

@@ -247,3 +247,35 @@ def test_which_products_the_own_kernels_take(dev, form, M, N, K, own):
     after = ops.gemm_info()
     assert after["tuned"] - before["tuned"] == own
     assert after["plans"] - before["plans"] >= own
+
+
+def test_gelu_keeps_32_bits(dev):
+    """The GELU of the products' epilogue and its derivative over N(0, 3), against float64.
+    One rounding of a result is 2.4e-8 in the 2-norm (0.41 of 2^-24): the GELU may be two
+    of them off and the derivative, a sum of two terms, three. (exp and 1 - g with their
+    full rounding came to 3.6e-7 in the derivative.) Then the ends of the range: GELU is x
+    or nothing there, infinity included, its derivative 1 or 0."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(3)
+    M, N = 16384, 4
+    x = torch.empty((M, N), device=dev).normal_(0.0, 3.0, generator=g)
+    ends = torch.tensor([0.0, 14.0, 1e15, 1e30, float("inf"), -14.0, -1e15, -1e30], device=dev)
+    x[:2] = ends.view(2, 4)
+    y, act, gx = (torch.empty((M, N), device=dev) for _ in range(3))
+    ops.device_activation_backward(gx, torch.ones_like(x), x, 1, M, N)
+    a = x[2:].double().requires_grad_(True)
+    r = gelu64(a)
+    d, = torch.autograd.grad(r.sum(), a)
+    assert rel(gx[2:], d) < 7.3e-8
+    assert gx[:2].view(-1)[[0, 1, 2, 5, 6]].tolist() == [0.5, 1.0, 1.0, 0.0, 0.0]
+    w, b, zero = torch.eye(4, device=dev), torch.zeros(4, device=dev), torch.zeros((4, 4), device=dev)
+    for v in ends.tolist():
+        b[1] = v
+        ops.device_linear_activation_fused_forward(y[:4], act[:4], zero, w, b, True, 1, 4, 4, 4)
+        assert torch.equal(act[:4, 1], torch.clamp(y[:4, 1], min=0.0)) and torch.equal(y[:4, 1], b[1].expand(4))
+    x = torch.empty((M, N), device=dev).normal_(0.0, 3.0, generator=g)
+    ops.device_linear_activation_fused_forward(y, act, x, torch.eye(4, device=dev), torch.zeros(4, device=dev), True,
+                                               1, M, 4, N)
+    assert torch.equal(y, x)
+    assert rel(act, gelu64(x.double())) < 4.9e-8
