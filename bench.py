@@ -595,7 +595,7 @@ def ops_bench(args):
     m1, v1 = torch.zeros(n_params, device=dev), torch.zeros(n_params, device=dev)
     cases.append(("adamw_step", 1, "hbm", f4 * 7 * n_params,
                   lambda: ops.device_adamw_step(prm, grd, m1, v1, n_params, 6e-4, 0.9, 0.95, 1e-8, 0.1, 1, st)))
-    cases.append(("scale_and_clip_grad", 1, "hbm", f4 * 3 * n_params,
+    cases.append(("scale_and_clip_grad", 1, "hbm", f4 * n_params,  # nothing to clip: one read
                   lambda: ops.device_scale_and_clip_grad(grd, n_params, 1e9, 1, st)))
 
     # the attention op pair of one layer, for the step total

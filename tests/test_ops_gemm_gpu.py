@@ -123,6 +123,31 @@ def test_second_pass_where_few_lanes_overflow(dev, row, col):
     assert rel(y, r) < tol(K) and rel(y[part], r[part]) < tol(K)
 
 
+@pytest.mark.parametrize("M,K,N", [(90, 768, 1540), (2048, 772, 2308)])
+def test_non_finite_operands_of_the_transposed_forms(dev, M, K, N):
+    """The same for grad_y w^T (few rows, and tiles of split k) and x^T grad_y, all on
+    the library's own kernels at these sizes."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(8)
+    x, w, gy = (torch.empty(s, device=dev).normal_(0.0, 1.0, generator=g) for s in ((M, K), (K, N), (M, N)))
+    x[3, 5], gy[40, 7], gy[50, 1], w[100, 9] = np.inf, -np.inf, 3.4e38, np.nan
+    w[:, 1] *= 1e-3
+    x[50] *= 1e-3
+    gx, gw, gb = torch.empty((M, K), device=dev), torch.zeros((K, N), device=dev), torch.zeros(N, device=dev)
+    before = ops.gemm_info()["tuned"]
+    ops.device_linear_backward(gx, gw, gb, gy, x, w, 1, M, K, N)
+    assert ops.gemm_info()["tuned"] == before + 2
+    for y, r, k in ((gx, gy.double() @ w.double().t(), N), (gw, x.double().t() @ gy.double(), M)):
+        f = r.float()
+        assert torch.equal(torch.isnan(y), torch.isnan(f))
+        assert torch.equal(torch.isinf(y), torch.isinf(f))
+        assert torch.equal(y[torch.isinf(f)], f[torch.isinf(f)])
+        big = r.abs() > 1e30
+        for part in (torch.isfinite(f) & big, torch.isfinite(f) & ~big):
+            assert rel(y[part], r[part]) < tol(k)
+
+
 def test_captured_products_replay(dev):
     """A captured linear layer replayed between eager calls gives the eager
     results' values, and the same bits on every replay."""
