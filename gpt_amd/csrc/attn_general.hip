@@ -17,7 +17,11 @@
 // What bounds it: a wave's chain of memory round trips and MFMAs, 2048 cycles
 // a block of the forward at d = 128. B = 2, T = 250, H = 6, d = 128, forward
 // and backward: 19.2 ms with one thread per row, now 50 us (forward 11, dQ and D 16, dK and
-// dV 22).
+// dV 22). A full card, B = 8, T = 1024, H = 6, d = 128: 142 and 622 us (91 TFLOP/s and,
+// of five products, 52).
+// Rows off 16 bytes (4-byte loads) past d = 128 spill up to 450 registers a lane: B = 2,
+// T = 250, H = 6, d = 130 58 and 405 us, where d = 132 takes 14.6 and 44, and one thread
+// per row took 6.8 and 25 ms.
 #include "attn_common.h"
 #include "attn_kernels.h"
 

@@ -26,7 +26,8 @@ constexpr float kGeluD3 = 2.0f * 0.107032f;  // 2 * 3 * 0.044715 * sqrt(2/pi)
 __device__ __forceinline__ float gelu_rest(float x, float *q)
 {
     const float e = __builtin_amdgcn_exp2f(-fabsf(x * fmaf(kGeluE3, x * x, kGeluE)));
-    *q = 1.0f / (1.0f + e);
+    const float d = 1.0f + e, i = __builtin_amdgcn_rcpf(d);
+    *q = fmaf(i, fmaf(-d, i, 1.0f), i);  // d in [1, 2]: one Newton step
     return e * *q;
 }
 
