@@ -189,20 +189,25 @@ __device__ __forceinline__ void embedding_bwd_wpe(float *__restrict__ gwpe, cons
 // (cpu_backend.cpp:102-117) without atomics. The other workgroups: grad_wpe.
 //
 // What bounds it: the commonest token's rows, added one after the other by one
-// workgroup; 16 rows' loads are in flight at once, since only the additions
-// have an order. 4096 rows of 768, ids as frequent as 1 / rank (the commonest
-// 262 times): 22 us, where one row's load at a time took 80, and grad_wpe 5.6 in
-// a launch of its own. Ids that hardly repeat leave the two searches, 23.5 us
-// (22.7 in two launches); with 32 counts per list instead of the waves' four
-// 30.0.
+// workgroup, with 12 rows' loads in flight at once, since only the additions
+// have an order; and where ids hardly repeat the searches, whose latency takes
+// waves to hide. Both want registers: 72 leave 7 waves a SIMD, with 32-bit
+// offsets in the list instead of 64-bit addresses (16 rows in 118 registers and 4
+// waves: uniform ids 25.9 us at 4096 rows of 768, 198 at 16384, now 19.8 and 125; one
+// row at a time, 8 waves 24.6 and 184). Ids as frequent as 1 / rank, the commonest
+// 262 of 4096 times: 19.9 us (16 rows 21.7, 8 rows 25, one row 82), grad_wpe's 5.6
+// in it; one id 4096 times 166. With 32 counts per list instead of the waves' four
+// 30.0 (of 25.9).
 template <bool V4>
-__global__ __launch_bounds__(256) void embedding_bwd_kernel(float *__restrict__ gwte, float *__restrict__ gwpe,
-                                                            const float *__restrict__ gy, const int *__restrict__ tok,
-                                                            int B, long rows, long tc, int C, int vocab_rows)
+__global__ __launch_bounds__(256, 6) void embedding_bwd_kernel(float *__restrict__ gwte, float *__restrict__ gwpe,
+                                                               const float *__restrict__ gy,
+                                                               const int *__restrict__ tok, int B, long rows,
+                                                               long tc, int C, int vocab_rows)
 {
-    constexpr int kPer = 8, kList = 256 * kPer, kFly = 16;
-    __shared__ int list[kList];
-    __shared__ int cnt[4];
+    constexpr int kPer = 8, kList = 256 * kPer, kFly = 12;
+    __shared__ unsigned list[kList];  // V4: byte offsets of the rows from the first listed
+    __shared__ int cnts[2][4];
+    int turn = 0;
     const long r = (long)blockIdx.y * gridDim.x + blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     if (r >= rows)
@@ -263,10 +268,15 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(float *__restrict__ 
                 mask[i] = __ballot(t[i] == id);
                 n += __popcll(mask[i]);
             }
+            // two sets of counts and one list: what writes one again comes after a
+            // barrier that everyone reaches after reading it
+            int *const cnt = cnts[turn++ & 1];
             if (lane == 0)
                 cnt[w] = n;
             __syncthreads();
             const int total = cnt[0] + cnt[1] + cnt[2] + cnt[3];
+            if (!total)
+                continue;
             int at = 0;
             for (int k = 0; k < w; ++k)
                 at += cnt[k];
@@ -276,14 +286,18 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(float *__restrict__ 
                 for (int i = 0; i < kPer; ++i)
                 {
                     if (t[i] == id)
-                        list[at + __popcll(mask[i] & ((1ull << lane) - 1ull))] = first + 64 * i;
+                        list[at + __popcll(mask[i] & ((1ull << lane) - 1ull))] =
+                            (unsigned)(first + 64 * i) * (V4 ? 4u * C : 1u);
                     at += __popcll(mask[i]);
                 }
             }
             __syncthreads();
             if (own)
             {
-                const float *src = gy + q0 * C + c;
+                const float *const src = gy + q0 * C;
+                const auto row4 = [&](unsigned at4) {
+                    return *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(src) + (at4 + 4u * c));
+                };
                 int j = 0;
                 if (V4)
                 {
@@ -292,7 +306,7 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(float *__restrict__ 
                         float4 v[kFly];
 #pragma unroll
                         for (int u = 0; u < kFly; ++u)
-                            v[u] = *reinterpret_cast<const float4 *>(src + (long)list[j + u] * C);
+                            v[u] = row4(list[j + u]);
 #pragma unroll
                         for (int u = 0; u < kFly; ++u)
                             acc4 = add4(acc4, v[u]);
@@ -302,21 +316,20 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(float *__restrict__ 
                         float4 v[4];
 #pragma unroll
                         for (int u = 0; u < 4; ++u)
-                            v[u] = *reinterpret_cast<const float4 *>(src + (long)list[j + u] * C);
+                            v[u] = row4(list[j + u]);
 #pragma unroll
                         for (int u = 0; u < 4; ++u)
                             acc4 = add4(acc4, v[u]);
                     }
                     for (; j < total; ++j)
-                        acc4 = add4(acc4, *reinterpret_cast<const float4 *>(src + (long)list[j] * C));
+                        acc4 = add4(acc4, row4(list[j]));
                 }
                 else
                 {
                     for (; j < total; ++j)
-                        acc += src[(long)list[j] * C];
+                        acc += src[(long)list[j] * C + c];
                 }
             }
-            __syncthreads();
         }
         if (own)
         {
@@ -1119,7 +1132,8 @@ hipError_t launch_embedding_bwd(float *grad_wte, float *grad_wpe, const float *g
                                 int C, int vocab_rows, hipStream_t st)
 {
     const long rows = (long)B * T, tc = (long)T * C;
-    const bool v4 = C % 4 == 0 && al16(grad_wte) && al16(grad_wpe) && al16(gy);
+    // (a list's offsets have 32 bits: 2048 rows)
+    const bool v4 = C % 4 == 0 && C <= 1 << 19 && al16(grad_wte) && al16(grad_wpe) && al16(gy);
     const long wpe = ((v4 ? tc / 4 : tc) + 255) / 256;
     // below 2^32 threads along a dimension of a launch; both parts check their range
     const long n = rows + wpe, row = 1L << 23;

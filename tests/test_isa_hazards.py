@@ -318,3 +318,21 @@ def test_mfma_read_scanner():
     assert early_mfma_reads(text(lines, 3))[1] == []
     assert early_mfma_reads(text([l.replace("a11", "a12") for l in lines], 5))[1] == []
     assert len(early_mfma_reads(text(["v_mfma_f32_16x16x4_f32 v[0:3], v35, v9, v[0:3]", "ds_write_b32 v9, v2"], 0))[1]) == 1
+
+
+def test_embedding_backward_leaves_registers_for_six_waves(tmp_path):
+    """At most 80 VGPRs: where ids hardly repeat, the embedding backward is a search
+    whose latency only waves hide (118 registers, 4 waves a SIMD: 198 us at 16384 rows
+    against 125)."""
+    if not os.path.exists(LIBS[1]):
+        pytest.skip("library not built")
+    counts = []
+    for i, obj in enumerate(gfx950_code_objects(LIBS[1])):
+        f = tmp_path / f"{i}.o"
+        f.write_bytes(obj)
+        notes = subprocess.run([OBJDUMP.replace("objdump", "readelf"), "--notes", str(f)], capture_output=True, text=True,
+                               check=True).stdout
+        for k in notes.split("- .agpr_count")[1:]:
+            if "embedding_bwd_kernel" in k:
+                counts.append(int(re.search(r"\.vgpr_count:\s+(\d+)", k).group(1)))
+    assert len(counts) == 2 and max(counts) <= 80, counts

@@ -28,6 +28,31 @@ def test_embedding_backward_many_rows_per_token(dev, rows, C, V, ids):
     assert np.array_equal(dp.cpu().numpy().view(np.uint32), p.view(np.uint32))
 
 
+@pytest.mark.parametrize("C", [36, 768, 1540, 30])
+def test_embedding_backward_lists_between_empty_ones(dev, C):
+    """Ids that hardly repeat: of an id's lists of 2048 rows the first, the last or some
+    between are empty, and full groups of loads (12, then 4) end at, before and after
+    a list's end."""
+    import torch
+
+    rows = 5 * 2048 + 77
+    tok = np.arange(rows, dtype=np.int32)
+    for id, at in enumerate(([0, 4096, 10316], [1, 2047, 2048, 8191], list(range(7, 7 + 2 * 11, 2)),
+                             list(range(100, 112)), list(range(2040, 2053)), list(range(2 * 2048, 3 * 2048, 73)),
+                             [9000] + list(range(9001, 9029)))):
+        tok[at] = rows + id
+    V = rows + 7
+    r = np.random.default_rng(C)
+    gy, w0 = (r.standard_normal(s, dtype=np.float32) for s in ((rows, C), (V, C)))
+    p0 = np.zeros((rows, C), np.float32)
+    w, p = w0.copy(), p0.copy()
+    pyops.embedding_backward(w, p, gy, tok, 1, rows, C)
+    dw, dp, dg, dt = (torch.from_numpy(a).to(dev) for a in (w0, p0, gy, tok))
+    ops.device_embedding_backward(dw, dp, dg, dt, 1, rows, C, vocab_rows=V)
+    assert np.array_equal(dw.cpu().numpy().view(np.uint32), w.view(np.uint32))
+    assert np.array_equal(dp.cpu().numpy().view(np.uint32), p.view(np.uint32))
+
+
 def test_embedding_backward_more_rows_than_one_grid_dimension(dev):
     """2^23 + 5 rows, a launch of two dimensions. All ids but the last are out of
     range, which adds nothing to grad_wte (and leaves one search of the rows)."""
