@@ -208,6 +208,33 @@ def test_tiny_operands(dev, M, K, N, e):
     assert rel(gw, x.double().t() @ gt.double()) < tol(M)
 
 
+@pytest.mark.parametrize("M,K,N", [(77, 768, 768), (2050, 768, 2304), (4096, 3072, 768)])
+@pytest.mark.parametrize("at", [33, 300, 700])
+def test_tiny_rows_after_zeros(dev, M, K, N, at):
+    """Rows and columns that are zero up to k = at, then tiny, then ordinary or zero, among
+    rows of zeros: the look at their further steps."""
+    import torch
+
+    g = torch.Generator(device=dev).manual_seed(at)
+    x, w = (torch.empty(s, device=dev).normal_(0.0, 1.0, generator=g) for s in ((M, K), (K, N)))
+    b, y = torch.zeros(N, device=dev), torch.empty((M, N), device=dev)
+    x[M // 3] = 0
+    x[[M // 2, M // 4], :at] = 0
+    x[M // 2] *= 2.0 ** -118
+    w[:, N // 3] = 0
+    w[:at, [N // 2, N // 4]] = 0
+    w[:, N // 4] *= 2.0 ** -118
+    ops.device_linear_activation_fused_forward(y, None, x, w, b, False, 1, M, K, N)
+    r = x.double() @ w.double()
+    assert not y[M // 3].any() and not y[:, N // 3].any()
+    rest = [n for n in range(N) if n != N // 4]
+    assert rel(y[:, rest], r[:, rest]) < tol(K)
+    assert rel(y[M // 2][rest], r[M // 2][rest]) < tol(K)
+    assert rel(y[M // 4][rest], r[M // 4][rest]) < tol(K)
+    rows = [m for m in range(M) if m != M // 2]
+    assert rel(y[rows, N // 4], r[rows, N // 4]) < tol(K)
+
+
 @pytest.mark.parametrize("form", ["nn", "nt"])
 @pytest.mark.parametrize("M,K,N", [(77, 3072, 768), (512, 768, 768), (128, 768, 2304), (4096, 768, 2304)])
 def test_errors_do_not_add_up_over_rows(dev, M, K, N, form):
